@@ -225,8 +225,9 @@ int motif_rope_split4_scaled(const void* q, const void* k, const void* v, void* 
                              int origin_first, void* stream);
 
 /* ------------------------------------------------------------------------ *
- * A GDA layer's prefill chunk from the projection outputs, in one attention
- * launch (plus the split merge when its rows are split).  Replaces, for a
+ * A GDA layer's prefill chunk from the projection outputs: one launch for
+ * RoPE and the chunk's cache rows, one for the attention of both passes (plus
+ * the split merge when its rows are split).  Replaces, for a
  * chunk of S tokens at cache offset `offset`, the rope calls on q and k
  * (src/mlx_motif/model.py:590-594), the 4-slot split with
  * update_and_fetch_4 (model.py:620-629, cache.py:337) and the four

@@ -61,12 +61,12 @@ int launch_sdpa_prefill_f16(const SdpaArgs& a, int waves, int ncb, int nblocks, 
 int launch_sdpa_prefill_bf16(const SdpaArgs& a, int waves, int ncb, int nblocks, hipStream_t s);
 int launch_sdpa_prefill_f32(const SdpaArgs& a, int waves, int ncb, int nblocks, hipStream_t s);
 
-// A GDA layer's prefill chunk from the projection outputs (RoPE, the
-// chunk's cache rows and both dual-V passes in one launch); f16 and bf16
-// instances have a kernel (head_dim 128).
-int launch_gda_prefill_proj_f16(const SdpaArgs& a, int waves, int ncb, int nblocks, hipStream_t s);
-int launch_gda_prefill_proj_bf16(const SdpaArgs& a, int waves, int ncb, int nblocks, hipStream_t s);
-int launch_gda_prefill_proj_f32(const SdpaArgs& a, int waves, int ncb, int nblocks, hipStream_t s);
+// RoPE, head split and 4-slot write (rope.hip) with q1 / q2 rows q_stride
+// elements apart (D; 2 D needs 16-bit values, D = 128 and 16-byte pointers).
+int launch_rope_split4(const void* q, const void* k, const void* v, void* q1, void* q2, void* k1,
+                       void* k2, void* v1, void* v2, int dtype, int B, int S, int q_groups, int gr,
+                       int k_groups, int kr, int D, int cap, int row0, int pos0, float theta,
+                       float position_scale, int origin_first, int q_stride, hipStream_t stream);
 
 // Pointer alignment (bytes) the kernels need for head dim D.
 int sdpa_fp_align(int dtype, int D);

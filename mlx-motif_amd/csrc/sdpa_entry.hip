@@ -171,6 +171,8 @@ static int sdpa_fp_run(const char* name, const void* q, const void* k, const voi
       aligned(v2, 16)) {
     const PrefillPlan pp = plan_prefill(B, Hq, Hkv, S_q, kv_len, D);
     a.nchunk = pp.nqb;
+    a.nqb_origin = pp.nqb;
+    a.q_stride = D;
     a.nsplit = pp.nsplit;
     a.rows_per_split = pp.rows_per_split;
     // Chunks (64+ virtual heads per KV head) deal their tiles to the splits
@@ -1105,9 +1107,8 @@ int motif_gda_prefill_proj_scaled(const void* q_proj, const void* k_proj, const 
   const int G_o = Hq_o / k_groups, G_n = q_groups / k_groups;
   const GdaPrefillPlan pp = plan_gda_prefill(B, k_groups, G_o, G_n, S, kv_len);
   SdpaArgs a{};
-  a.q = q_proj;
+  a.q = y_origin; a.q2 = y_noise; a.q_stride = 2 * D;  // q roped into the rows of y, below
   a.k = k1; a.k2 = k2; a.v1 = v1; a.v2 = v2;
-  a.new_k1 = k_proj; a.new_v1 = v_proj;
   a.y = y_origin;
   a.y2 = y_noise;
   a.B = B; a.Hq = Hq_o; a.Hkv = k_groups; a.S_q = S;
@@ -1118,10 +1119,7 @@ int motif_gda_prefill_proj_scaled(const void* q_proj, const void* k_proj, const 
   a.nsplit = pp.nsplit; a.rows_per_split = pp.rows_per_split;
   a.fused_merge = 0;
   a.qscale = scale * 1.4426950408889634f;
-  a.q_groups = q_groups; a.q_gr = gr; a.q_origin_first = origin_first != 0;
-  a.rope_log2_theta = log2f(theta);
-  a.rope_pos_scale = position_scale;
-  a.rope_pos0 = offset;
+  a.tiles_rr = 1;
   a.y2_row0 = (long)B * Hq_o * S;
   if (pp.nsplit > 1) {
     const int rc = carve_split_ws(name, a, workspace, workspace_bytes,
@@ -1133,9 +1131,22 @@ int motif_gda_prefill_proj_scaled(const void* q_proj, const void* k_proj, const 
   int rc = check_partials(name, a, false);
   if (rc != MOTIF_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
+  // Two launches: RoPE, the split and the chunk's cache rows, then the
+  // attention of both passes over the cache.  RoPE inside the attention
+  // launch bound it: each of a first 512-row chunk's 20 query blocks per KV
+  // head computed the angles of its q rows and of every K tile again.  One
+  // layer's pass with its epilogue (32 + 8 heads over 8 KV heads), RoPE inside
+  // / in a launch of its own: 512 rows at offset 0, bf16, 52.0 / 34.0 us;
+  // 2048 rows at offset 6150, fp16, 736 / 650 us.  The roped q needs no
+  // scratch: row r of q goes into the first half of row r of y, which only
+  // the workgroups of that row read before the row's result replaces it.
+  rc = launch_rope_split4(q_proj, k_proj, v_proj, y_origin, y_noise, k1, k2, v1, v2, dtype, B, S,
+                          q_groups, gr, k_groups, 1, D, kv_cap, offset, offset, theta,
+                          position_scale, origin_first, 2 * D, s);
+  if (rc != MOTIF_OK) return rc;
   const int nblocks = sdpa_grid_blocks(B * k_groups, a.nchunk, pp.nsplit);
-  rc = dtype == MOTIF_F16 ? launch_gda_prefill_proj_f16(a, pp.waves, pp.ncb, nblocks, s)
-                              : launch_gda_prefill_proj_bf16(a, pp.waves, pp.ncb, nblocks, s);
+  rc = dtype == MOTIF_F16 ? launch_sdpa_prefill_f16(a, pp.waves, pp.ncb, nblocks, s)
+                          : launch_sdpa_prefill_bf16(a, pp.waves, pp.ncb, nblocks, s);
   if (rc != MOTIF_OK || pp.nsplit == 1) return rc;
   // One merge over both passes' partial rows (noise rows into y_noise).
   SdpaArgs m = a;

@@ -135,18 +135,6 @@ int MOTIF_CAT(launch_sdpa_prefill_, MOTIF_SUFFIX)(const SdpaArgs& a, int waves, 
   return MOTIF_ERR_UNSUPPORTED;
 }
 
-// Prefill chunk of a GDA layer from the projections (fp16 or bf16, head_dim
-// 128).
-int MOTIF_CAT(launch_gda_prefill_proj_, MOTIF_SUFFIX)(const SdpaArgs& a, int waves, int ncb,
-                                                     int nblocks, hipStream_t s) {
-  if constexpr (std::is_same<MOTIF_ELEM, half_t>::value ||
-                std::is_same<MOTIF_ELEM, bf16_t>::value) {
-    return launch_gda_prefill_proj_16<MOTIF_ELEM>(a, waves, ncb, nblocks, s);
-  }
-  set_error("gda_prefill_proj: no variant for this element type");
-  return MOTIF_ERR_UNSUPPORTED;
-}
-
 // Same over the packed q4/q8 cache (fp16 scales, head_dim 128).
 int MOTIF_CAT(launch_gda_decode_q_, MOTIF_SUFFIX)(const SdpaArgs& a, int bits, int gc, int nblocks,
                                                  hipStream_t s) {

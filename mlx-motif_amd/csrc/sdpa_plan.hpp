@@ -86,20 +86,17 @@ struct SdpaArgs {
   int q_origin_first;
   float rope_log2_theta;
   float rope_pos_scale = 1.f;  // RoPE position scale: 1, or 1 / factor (linear scaling)
-  // Prefill chunk of a GDA layer from the projection outputs
-  // (gda_prefill_proj_kernel): q is q_proj (B, S_q, q_groups*(q_gr+1)*D),
-  // new_k1 k_proj and new_v1 v_proj (B, S_q, 2*Hkv*D; k1[g] = head 2g,
-  // k2[g] = 2g+1, likewise v1/v2).  Query blocks [0, nqb_origin) of a
-  // (b, KV head, split) run the origin pass (G heads per KV head: q1 x k1,
-  // output y), the others the noise pass (G2 heads: q2 x k2, output y2,
-  // whose split partials start at row y2_row0).  The chunk is cache rows
-  // kv_len - S_q .. kv_len - 1, roped at positions rope_pos0 + s.
+  // Shared-tile multi-row kernel: rows of q are q_stride elements apart (D,
+  // or 2 D where the roped q of a GDA layer's chunk sits in the rows of y it
+  // becomes).  Query blocks [0, nqb_origin) of a (b, KV head, split) run the
+  // origin pass (G heads per KV head: q x k, output y), the others a layer's
+  // noise pass (G2 heads: q2 x k2, output y2, whose split partials start at
+  // row y2_row0).
+  int q_stride;
   void* y2;
   long y2_row0;
   int nqb_origin;
   int G2;  // noise heads per KV head (the prefill chunk and the fused decode step)
-  int q_groups, q_gr;
-  int rope_pos0;
 };
 
 struct SdpaPlan {
@@ -156,8 +153,8 @@ struct PrefillPlan {
 };
 PrefillPlan plan_prefill(int B, int Hq, int Hkv, int S_q, int kv_len, int D);
 
-// Plan of a GDA layer's prefill chunk from the projections
-// (gda_prefill_proj_kernel): per (b, KV head) nqb_origin query blocks of the
+// Plan of the attention launch of a GDA layer's prefill chunk
+// (motif_gda_prefill_proj): per (b, KV head) nqb_origin query blocks of the
 // origin pass (G_origin heads x S rows) and nqb_noise of the noise pass
 // (G_noise heads x S rows) of waves x 16 virtual heads each; rows are split
 // (to about one workgroup per CU) only when the blocks fill fewer than half
