@@ -39,6 +39,11 @@ bool qpair_bf16_ok(const SdpaArgs& a, int D, int gs, int bits);
 int launch_sdpa_qslab(const SdpaArgs& a, int bits, int gs, int ncb, int waves, int nblocks,
                       hipStream_t s);
 
+// Prompt chunks over the packed cache (sdpa_qprefill.hip); fp16 or bf16 q,
+// scales and y, plan_prefill's waves and column blocks.
+int launch_sdpa_qprefill(const SdpaArgs& a, bool bf16, int bits, int waves, int ncb, int nblocks,
+                         hipStream_t st);
+
 // Split merge (second launch when a.fused_merge == 0 and nsplit > 1) for
 // outputs of the given element type.
 int launch_sdpa_merge_f16(const SdpaArgs& a, int D, hipStream_t s);

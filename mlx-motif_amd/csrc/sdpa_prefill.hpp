@@ -235,6 +235,29 @@ struct SwizzledTileAcc {
   __device__ __forceinline__ void store(const SdpaArgs& a, long vrow, int split, int blk) const {
     store_to(a.y, vrow, a.part_o, a.part_ml, vrow, a.nsplit, split, blk, a.part_f16);
   }
+  // The normalised result into row yrow of y, as elements of type O.
+  template <typename O>
+  __device__ __forceinline__ void store_y(void* y, long yrow, int blk) const {
+    constexpr int D = 128;
+    const float l = accl[0];
+    const float inv = l == 0.f ? 1.f : 1.f / l;  // o stays 0 when no key is visible
+    uint16_t* yp = (uint16_t*)y + yrow * 2 * D + 32 * blk;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {  // channels 32*blk + 8*p .. +7
+      uint32_t w1[4], w2[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int j = 2 * p + t / 2;
+        const int r = 2 * (t % 2);
+        w1[t] = (uint32_t)Elem<O>::from_f32(acc1[j][r] * inv) |
+                ((uint32_t)Elem<O>::from_f32(acc1[j][r + 1] * inv) << 16);
+        w2[t] = (uint32_t)Elem<O>::from_f32(acc2[j][r] * inv) |
+                ((uint32_t)Elem<O>::from_f32(acc2[j][r + 1] * inv) << 16);
+      }
+      *reinterpret_cast<uint4*>(yp + 8 * p) = make_uint4(w1[0], w1[1], w1[2], w1[3]);
+      *reinterpret_cast<uint4*>(yp + D + 8 * p) = make_uint4(w2[0], w2[1], w2[2], w2[3]);
+    }
+  }
   // The same into row yrow of y (nsplit == 1) or partial row prow (fp32 o,
   // or fp16 o / l with f16).
   __device__ __forceinline__ void store_to(void* y, long yrow, float* part_o, float* part_ml,
@@ -243,23 +266,7 @@ struct SwizzledTileAcc {
     constexpr int D = 128;
     const float l = accl[0];
     if (nsplit == 1) {
-      const float inv = l == 0.f ? 1.f : 1.f / l;  // o stays 0 when no key is visible
-      uint16_t* yp = (uint16_t*)y + yrow * 2 * D + 32 * blk;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {  // channels 32*blk + 8*p .. +7
-        uint32_t w1[4], w2[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int j = 2 * p + t / 2;
-          const int r = 2 * (t % 2);
-          w1[t] = (uint32_t)Elem<T>::from_f32(acc1[j][r] * inv) |
-                  ((uint32_t)Elem<T>::from_f32(acc1[j][r + 1] * inv) << 16);
-          w2[t] = (uint32_t)Elem<T>::from_f32(acc2[j][r] * inv) |
-                  ((uint32_t)Elem<T>::from_f32(acc2[j][r + 1] * inv) << 16);
-        }
-        *reinterpret_cast<uint4*>(yp + 8 * p) = make_uint4(w1[0], w1[1], w1[2], w1[3]);
-        *reinterpret_cast<uint4*>(yp + D + 8 * p) = make_uint4(w2[0], w2[1], w2[2], w2[3]);
-      }
+      store_y<T>(y, yrow, blk);
     } else if (f16) {
       const int ns = nsplit;
       const float inv = l == 0.f ? 0.f : 1.f / l;
