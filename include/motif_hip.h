@@ -280,6 +280,12 @@ int motif_quantize(const void* x, uint32_t* data, void* scales, void* biases, in
  * dequant bridge (cache.py:448-465). */
 int motif_dequantize(const uint32_t* data, const void* scales, const void* biases, void* y,
                      int dtype, int64_t rows, int D, int bits, int group_size, void* stream);
+/* The same for rows [0,rows) of the four slots of a packed cache of capacity
+ * kv_cap (laid out as for motif_quant_write4) in one dispatch: y[i]
+ * (B,H,rows,D) dtype. */
+int motif_dequantize4(const uint32_t* const data[4], const void* const scales[4],
+                      const void* const biases[4], void* const y[4], int dtype, int B, int H,
+                      int rows, int D, int kv_cap, int bits, int group_size, void* stream);
 
 /* ------------------------------------------------------------------------ *
  * Batched 4-slot quantised cache write in ONE dispatch: quantise rows

@@ -76,23 +76,64 @@ __global__ void __launch_bounds__(256) quant_write4_kernel(Write4Args a) {
   }
 }
 
-// y = T(float(scale) * float(u) + float(bias)), one thread per value.
-template <typename T, int BITS>
-__global__ void __launch_bounds__(256) dequantize_kernel(const uint32_t* data, const void* scales,
-                                                         const void* biases, void* y, long n,
-                                                         int D, int gs) {
+struct DequantArgs {
+  const uint32_t* data[4];  // (bh, cap, D*bits/32) per slot
+  const void* scales[4];    // (bh, cap, D/gs)
+  const void* biases[4];
+  void* y[4];               // (bh, n, D): rows [0, n) of each bh
+  int64_t chunks;           // bh * n * D / 8 per slot
+  int64_t n, cap;
+  int D, gs;
+};
+
+// y = T(float(scale) * float(u) + float(bias)): one thread per 8 values
+// (one 16-byte store of 16-bit values), one grid row per slot.  Bound by its
+// bytes, of which the values written are the most; one thread per value
+// (2-byte stores, a 64-bit division each) took 10.2 us for a slot of 8 x 3204
+// rows from 4-bit codes (and the wrapper's slices three copies a slot: the
+// bridge's whole pass 209 -> 139 us).
+// I: index type (32 bits unless a slot has 2^32 chunks).
+template <typename T, int BITS, typename I>
+__global__ void __launch_bounds__(256) dequantize_kernel(DequantArgs a) {
 #pragma clang fp contract(off)
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  constexpr int EL = 32 / BITS;
-  const long row = i / D;
-  const int c = (int)(i % D);
-  const uint32_t word = data[row * (D / EL) + c / EL];
-  const uint32_t u = (word >> ((c % EL) * BITS)) & ((1u << BITS) - 1u);
-  const long si = row * (D / gs) + c / gs;
-  const float s = Elem<T>::load(scales, si);
-  const float b = Elem<T>::load(biases, si);
-  Elem<T>::store(y, i, s * (float)u + b);
+  typedef uint32_t u32x2_t __attribute__((ext_vector_type(2), aligned(4)));
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4), aligned(2)));
+  const I i = (I)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (I)a.chunks) return;
+  const int slot = blockIdx.y;
+  const I cpr = (I)(a.D / 8);  // chunks per row
+  const I row = i / cpr;
+  const int c = (int)(i % cpr);
+  const long crow = (long)(row / (I)a.n) * a.cap + (long)(row % (I)a.n);
+  uint32_t w[2];
+  if constexpr (BITS == 8) {
+    const u32x2_t x = *reinterpret_cast<const u32x2_t*>(a.data[slot] + crow * (a.D / 4) + 2 * c);
+    w[0] = x.x;
+    w[1] = x.y;
+  } else {
+    w[0] = a.data[slot][crow * (a.D / 8) + c];
+  }
+  const long si = crow * (a.D / a.gs) + 8 * c / a.gs;
+  const float s = Elem<T>::load(a.scales[slot], si);
+  const float b = Elem<T>::load(a.biases[slot], si);
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t u = BITS == 8 ? (w[e / 4] >> (8 * (e % 4))) & 0xFFu : (w[0] >> (4 * e)) & 0xFu;
+    v[e] = s * (float)u + b;
+  }
+  const long yi = (long)row * a.D + 8 * c;
+  if constexpr (Elem<T>::kBytes == 2) {
+    uint32_t h[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      h[p] = (uint32_t)Elem<T>::from_f32(v[2 * p]) | ((uint32_t)Elem<T>::from_f32(v[2 * p + 1]) << 16);
+    *reinterpret_cast<u32x4_t*>((uint16_t*)a.y[slot] + yi) = u32x4_t{h[0], h[1], h[2], h[3]};
+  } else {
+    u32x4_t* yp = reinterpret_cast<u32x4_t*>((float*)a.y[slot] + yi);
+    yp[0] = __builtin_bit_cast(u32x4_t, make_float4(v[0], v[1], v[2], v[3]));
+    yp[1] = __builtin_bit_cast(u32x4_t, make_float4(v[4], v[5], v[6], v[7]));
+  }
 }
 
 // ----------------------------------------------------------------- host ---
@@ -163,10 +204,12 @@ struct Write4Op {
 
 template <typename T, int BITS>
 struct DequantOp {
-  static void run(const uint32_t* d, const void* s, const void* b, void* y, long n, int D,
-                  int gs, hipStream_t st) {
-    const unsigned blocks = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL((dequantize_kernel<T, BITS>), blocks, 256, 0, st, d, s, b, y, n, D, gs);
+  static void run(const DequantArgs& a, int slots, hipStream_t st) {
+    const dim3 grid((unsigned)((a.chunks + 255) / 256), (unsigned)slots);
+    if (a.chunks < (1LL << 32) - 256)
+      hipLaunchKernelGGL((dequantize_kernel<T, BITS, uint32_t>), grid, dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((dequantize_kernel<T, BITS, int64_t>), grid, dim3(256), 0, st, a);
   }
 };
 
@@ -205,9 +248,40 @@ int motif_dequantize(const uint32_t* data, const void* scales, const void* biase
   MOTIF_REQUIRE(rows >= 0, "dequantize: rows=%lld must be >= 0", (long long)rows);
   if (rows == 0) return MOTIF_OK;
   MOTIF_REQUIRE(data && scales && biases && y, "dequantize: null tensor pointer");
-  by_type_bits<DequantOp>(dtype, bits, data, scales, biases, y, (long)rows * D, D, group_size,
-                          (hipStream_t)stream);
+  DequantArgs a{};
+  a.data[0] = data; a.scales[0] = scales; a.biases[0] = biases; a.y[0] = y;
+  a.chunks = rows * (D / 8);
+  a.n = a.cap = rows;
+  a.D = D;
+  a.gs = group_size;
+  by_type_bits<DequantOp>(dtype, bits, a, 1, (hipStream_t)stream);
   return check_launch("dequantize");
+}
+
+int motif_dequantize4(const uint32_t* const data[4], const void* const scales[4],
+                      const void* const biases[4], void* const y[4], int dtype, int B, int H,
+                      int rows, int D, int kv_cap, int bits, int group_size, void* stream) {
+  CallScope scope;
+  clear_error();
+  int rc = quant_checks("dequantize4", dtype, D, bits, group_size);
+  if (rc != MOTIF_OK) return rc;
+  MOTIF_REQUIRE(B >= 1 && H >= 1, "dequantize4: B and H must be >= 1");
+  MOTIF_REQUIRE(rows >= 0 && rows <= kv_cap, "dequantize4: rows=%d must be in [0, %d]", rows,
+                kv_cap);
+  if (rows == 0) return MOTIF_OK;
+  MOTIF_REQUIRE(data && scales && biases && y, "dequantize4: null slot array");
+  DequantArgs a{};
+  for (int i = 0; i < 4; ++i) {
+    MOTIF_REQUIRE(data[i] && scales[i] && biases[i] && y[i], "dequantize4: null pointer");
+    a.data[i] = data[i]; a.scales[i] = scales[i]; a.biases[i] = biases[i]; a.y[i] = y[i];
+  }
+  a.chunks = (int64_t)B * H * rows * (D / 8);
+  a.n = rows;
+  a.cap = kv_cap;
+  a.D = D;
+  a.gs = group_size;
+  by_type_bits<DequantOp>(dtype, bits, a, 4, (hipStream_t)stream);
+  return check_launch("dequantize4");
 }
 
 int motif_quant_write4(const void* k1, const void* k2, const void* v1, const void* v2,

@@ -75,6 +75,7 @@ _SIGNATURES = {
     ),
     "motif_quantize": (_c_int, [_vp] * 4 + [_c_int, _c_i64, _c_int, _c_int, _c_int, _vp]),
     "motif_dequantize": (_c_int, [_vp] * 4 + [_c_int, _c_i64, _c_int, _c_int, _c_int, _vp]),
+    "motif_dequantize4": (_c_int, [_VP4] * 4 + [_c_int] * 8 + [_vp]),
     "motif_quant_write4": (
         _c_int,
         [_vp] * 4 + [_VP4, _VP4, _VP4] + [_c_int] * 9 + [_vp],

@@ -191,6 +191,9 @@ class MotifGroupedQuantizedKVCache(MotifGroupedKVCacheBase):
         (the dequant bridge of ``cache.py:448-465``)."""
         self._update_4(k1, k2, v1, v2)
         o = self.offset
+        slots = (self.k1, self.k2, self.v1, self.v2)
+        if not _common._DISABLE and self._uniform(slots, D := k1.shape[-1]):
+            return self._dequantize_native(slots, o, D)
 
         def _deq(slot):
             return dequantize(
@@ -199,6 +202,33 @@ class MotifGroupedQuantizedKVCache(MotifGroupedKVCacheBase):
             )
 
         return _deq(self.k1), _deq(self.k2), _deq(self.v1), _deq(self.v2)
+
+    def _uniform(self, slots, D: int) -> bool:
+        """Whether the slots are whole row-contiguous buffers of one type and
+        shape (a restored state may hold views)."""
+        lead, dtype = slots[0][0].shape[:3], slots[0][1].dtype
+        data, groups = (*lead, D * self.bits // 32), (*lead, D // self.group_size)
+        return all(d.is_contiguous() and s.is_contiguous() and b.is_contiguous()
+                   and d.shape == data and s.shape == groups and b.shape == groups
+                   and d.dtype == torch.uint32 and s.dtype == dtype and b.dtype == dtype
+                   for d, s, b in slots)
+
+    def _dequantize_native(self, slots, rows: int, D: int):
+        """The four slots' live rows in one ``motif_dequantize4`` dispatch,
+        read where they lie."""
+        B, H, cap, _ = slots[0][0].shape
+        dtype = slots[0][1].dtype
+        dev = _native.require_device(*(x for s in slots for x in s))
+        out = tuple(torch.empty((B, H, rows, D), dtype=dtype, device=dev) for _ in slots)
+        vp4 = _native._VP4
+        _native.check(
+            _native.lib().motif_dequantize4(
+                *[vp4(*[s[i].data_ptr() for s in slots]) for i in range(3)],
+                vp4(*[t.data_ptr() for t in out]), _native.dtype_code(dtype), B, H, rows, D, cap,
+                self.bits, self.group_size, _native.stream_of(dev),
+            )
+        )
+        return out
 
     def update_and_fetch_4_quantized(self, k1, k2, v1, v2):
         """Quantise + append; return each slot's FULL capacity triple for
