@@ -78,6 +78,22 @@ static void update_tuning(F f) {
 
 static size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// Row splits for `units` workgroup columns on a GPU that runs `slots` of
+// their workgroups at once: the most that stay within one round, since a
+// second round of a few workgroups takes about as long as the first (fused
+// fp16 decode step, 32 + 8 heads over 8 KV heads, batch 5 over 12000 rows:
+// 7 splits, 280 workgroups, 124.6 us; 6 splits, 240, 87.7 us).  Two full
+// rounds where they fill the GPU so much better that each round is at least a
+// seventh shorter (batch 12 over 5330 rows, 2 / 3 / 5 splits: 105 / 127 / 93
+// us; batch 7, a ninth shorter: 4 / 5 / 9 splits 97 / 131 / 90 us in fp16,
+// 50 / 70 / 52 us for bf16 over q4) and there are at most max_two splits.
+static int fill_splits(long units, long slots, long max_two) {
+  if (units >= slots) return 1;
+  const long one = slots / units;
+  const long two = 2 * slots / units;
+  return (int)(7 * 2 * one <= 6 * two && two <= max_two ? two : one);
+}
+
 SdpaPlan plan_sdpa(int B, int Hq, int Hkv, int S_q, int kv_len, int D, int gc_max,
                    int waves_pref, int wgs_per_cu, int gc_fixed) {
   SdpaPlan p{};
@@ -112,7 +128,11 @@ SdpaPlan plan_sdpa(int B, int Hq, int Hkv, int S_q, int kv_len, int D, int gc_ma
   if (tuning().rows_per_split > 0) {
     rps = (int)round_up((size_t)tuning().rows_per_split, 16);  // whole 16-row tiles
   } else {
-    int nsplit = (min_wgs + units - 1) / units;
+    // Two rounds only while the partials stay small (7 MiB: they are merged in
+    // a launch that reads them all, and the no-alloc scratch holds 8).
+    const long max_two = (7L << 20) / ((long)B * Hq * S_q * (2 * D + 2) * (long)sizeof(float));
+    int nsplit = tuning().min_wgs > 0 ? (min_wgs + units - 1) / units
+                                      : fill_splits(units, min_wgs, max_two);
     int max_split = (rows + step - 1) / step;  // at least one iteration each
     if (nsplit > max_split) nsplit = max_split;
     if (nsplit < 1) nsplit = 1;
@@ -173,7 +193,12 @@ PrefillPlan plan_prefill(int B, int Hq, int Hkv, int S_q, int kv_len, int D) {
   p.nqb = (GV + cols - 1) / cols;
   const long units = (long)bh * p.nqb;
   const int rows = kv_len > 0 ? kv_len : 1;
-  int nsplit = units >= cus ? 1 : (int)((cus + units - 1) / units);
+  // Two rounds need splits of 512+ rows (333 rows of 32 heads over 8, 88 query
+  // blocks: over 3204 rows 2 / 3 / 5 splits 65.1 / 75.7 / 60.9 us, over 1100
+  // rows 34.1 / 41.2 / 38.3) and partials of at most 64 MiB.
+  const long max_two =
+      std::min<long>(rows / 512, (64L << 20) / ((long)B * Hq * S_q * 2 * D * (long)sizeof(float)));
+  int nsplit = fill_splits(units, cus, max_two);
   const int max_split = (rows + 127) / 128;  // at least 128 rows per split
   if (nsplit > max_split) nsplit = max_split;
   if (nsplit > kMaxSplits) nsplit = kMaxSplits;
@@ -252,7 +277,7 @@ QSlabPlan plan_qslab(int B, int Hq, int Hkv, int S_q, int kv_len, int D) {
   const long units = (long)B * Hkv * p.nchunk;
   const int rows = kv_len > 0 ? kv_len : 1;
   const int cus = tuning().min_wgs > 0 ? tuning().min_wgs : device_cu_count();
-  int nsplit = units >= cus ? 1 : (int)((cus + units - 1) / units);
+  int nsplit = tuning().min_wgs > 0 ? (int)((cus + units - 1) / units) : fill_splits(units, cus, 0);
   const int max_split = (rows + step - 1) / step;  // at least one step each
   if (nsplit > max_split) nsplit = max_split;
   if (nsplit > kMaxSplits) nsplit = kMaxSplits;
