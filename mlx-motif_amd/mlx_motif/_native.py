@@ -204,14 +204,14 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "mlx_motif HIP kernels need tensors on a ROCm device "
                 f"(got {t.device}); set MLX_MOTIF_DISABLE_KERNELS=1 for the reference path"
             )
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
     return dev
 
@@ -220,8 +220,13 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def _index(device: torch.device) -> int:
+    return device.index if device.index is not None else torch.cuda.current_device()
+
+
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle alone: a torch.cuda.Stream object costs a few times the lookup
+    return torch._C._cuda_getCurrentRawStream(_index(device))
 
 
 # ------------------------------------------------------------ workspace ---
@@ -243,8 +248,10 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     below the live buffer's size.  ``release_retired_workspaces`` frees it
     once no such graph is alive.
     """
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           stream_of(device))
+    key = (_index(device), stream_of(device))
+    buf = _workspaces.get(key)  # entries only ever grow: no lock to read one
+    if buf is not None and buf.numel() >= nbytes:
+        return buf
     with _ws_lock:
         buf = _workspaces.get(key)
         if buf is None or buf.numel() < nbytes:

@@ -25,9 +25,20 @@ def contiguous(t: torch.Tensor) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
+def as_param(t: torch.Tensor, device: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """``t`` row-contiguous on ``device`` in ``dtype``: itself where it is so."""
+    if t.dtype is dtype and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=dtype).contiguous()
+
+
 def f32_scalar_tensor(value, device: torch.device) -> torch.Tensor:
-    """A 1-element fp32 device tensor from a tensor or a Python number, without
-    a host synchronisation when it is already a device tensor."""
+    """A device tensor whose first element is ``value`` in fp32, from a tensor
+    or a Python number, without a host synchronisation when it is already a
+    device tensor."""
     if isinstance(value, torch.Tensor):
+        if (value.dtype is torch.float32 and value.device == device and value.is_contiguous()
+                and value.numel()):
+            return value
         return value.reshape(-1)[:1].to(device=device, dtype=torch.float32).contiguous()
     return torch.tensor([float(value)], dtype=torch.float32, device=device)

@@ -39,6 +39,7 @@ from . import _common
 from .attention import _q_contract, sdpa_dual_v_q4_reference, sdpa_dual_v_reference
 from .gda import gda_post_split_reference
 from .quant import quantize_reference
+from .rope import rope_position_scale, rope_split4, rope_split4_reference
 
 
 def gda_decode_attention_reference(q1, q2, k1, k2, v1, v2, scale: float, subln_weight,
@@ -158,7 +159,7 @@ def gda_decode_attention(q1, q2, k1, k2, v1, v2, scale: float, subln_weight, lam
         if t.dtype != q1.dtype:
             raise TypeError(f"dtype {t.dtype} must match q1 dtype {q1.dtype}")
     q1, q2, k1, k2, v1, v2 = (_common.contiguous(t) for t in (q1, q2, k1, k2, v1, v2))
-    w = subln_weight.to(device=dev, dtype=q1.dtype).contiguous()
+    w = _common.as_param(subln_weight, dev, q1.dtype)
     lam = _common.f32_scalar_tensor(lambda_full, dev)
     y = torch.empty((B, H_o, 1, 2 * D), dtype=q1.dtype, device=dev)
     lib = _native.lib()
@@ -237,7 +238,7 @@ def gda_decode_attention_q4(q1, q2, k1_q: tuple, k2_q: tuple, v1_q: tuple, v2_q:
         raise TypeError(f"q2 dtype {q2.dtype} must match q1 dtype {q1.dtype}")
     q1, q2 = _common.contiguous(q1), _common.contiguous(q2)
     slots = tuple(tuple(_common.contiguous(x) for x in t) for t in slots)
-    w = subln_weight.to(device=dev, dtype=q1.dtype).contiguous()
+    w = _common.as_param(subln_weight, dev, q1.dtype)
     lam = _common.f32_scalar_tensor(lambda_full, dev)
     y = torch.empty((B, H_o, 1, 2 * D), dtype=q1.dtype, device=dev)
     lib = _native.lib()
@@ -278,8 +279,6 @@ def gda_decode_attention_from_proj(q_proj, k_proj, v_proj, k1, k2, v1, v2, scale
     attention launch ropes and writes; then the merge); otherwise
     ``rope_split4`` followed by ``gda_decode_attention``.  ``rope_scaling``:
     None, or a default / linear config (``rope.rope_position_scale``)."""
-    from .rope import rope_position_scale, rope_split4, rope_split4_reference
-
     pscale = rope_position_scale(rope_scaling)
 
     B, S, nq = q_proj.shape
@@ -306,7 +305,7 @@ def gda_decode_attention_from_proj(q_proj, k_proj, v_proj, k1, k2, v1, v2, scale
         if t.dtype != q_proj.dtype:
             raise TypeError(f"dtype {t.dtype} must match q dtype {q_proj.dtype}")
     q_proj, k_proj, v_proj = (_common.contiguous(t) for t in (q_proj, k_proj, v_proj))
-    w = subln_weight.to(device=dev, dtype=q_proj.dtype).contiguous()
+    w = _common.as_param(subln_weight, dev, q_proj.dtype)
     lam = _common.f32_scalar_tensor(lambda_full, dev)
     y = torch.empty((B, H_kv * gr, 1, 2 * D), dtype=q_proj.dtype, device=dev)
     lib = _native.lib()
@@ -339,8 +338,6 @@ def gda_decode_attention_q4_from_proj(q_proj, k_proj, v_proj, k1_q: tuple, k2_q:
     shape, else ``rope_split4`` then ``gda_decode_attention_q4(new_kv=...)``
     (the same values bit for bit).  ``rope_scaling``: None, or a default /
     linear config."""
-    from .rope import rope_position_scale, rope_split4, rope_split4_reference
-
     pscale = rope_position_scale(rope_scaling)
 
     B, S, nq = q_proj.shape
@@ -367,7 +364,7 @@ def gda_decode_attention_q4_from_proj(q_proj, k_proj, v_proj, k1_q: tuple, k2_q:
     _require_in_place([x for t in slots for x in t])
     dev = _native.require_device(q_proj, k_proj, v_proj, *(x for t in slots for x in t))
     q_proj, k_proj, v_proj = (_common.contiguous(t) for t in (q_proj, k_proj, v_proj))
-    w = subln_weight.to(device=dev, dtype=q_proj.dtype).contiguous()
+    w = _common.as_param(subln_weight, dev, q_proj.dtype)
     lam = _common.f32_scalar_tensor(lambda_full, dev)
     y = torch.empty((B, H_kv * gr, 1, 2 * D), dtype=q_proj.dtype, device=dev)
     lib = _native.lib()

@@ -51,7 +51,7 @@ def gda_post_split(attn_o, attn_n, subln_weight, lambda_full, lambda_init: float
         raise TypeError(f"attn_n dtype {attn_n.dtype} must match attn_o dtype {attn_o.dtype}")
     o = _common.contiguous(attn_o)
     n = _common.contiguous(attn_n)
-    w = subln_weight.to(device=dev, dtype=attn_o.dtype).contiguous()
+    w = _common.as_param(subln_weight, dev, attn_o.dtype)
     lam = _common.f32_scalar_tensor(lambda_full, dev)
     y = torch.empty_like(o)
     _native.check(
@@ -76,7 +76,7 @@ def gda_post(merged, subln_weight, lambda_full, lambda_init: float, q_groups: in
     assert q_heads == q_origin + q_groups, f"q_heads={q_heads} expected {q_origin}+{q_groups}"
     dev = _native.require_device(merged)
     m = _common.contiguous(merged)
-    w = subln_weight.to(device=dev, dtype=merged.dtype).contiguous()
+    w = _common.as_param(subln_weight, dev, merged.dtype)
     lam = _common.f32_scalar_tensor(lambda_full, dev)
     y = torch.empty((B, q_origin, S, channels), dtype=merged.dtype, device=dev)
     _native.check(

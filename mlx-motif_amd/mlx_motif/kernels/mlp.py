@@ -41,8 +41,8 @@ def polynorm(x, weight, bias, eps: float = 1e-6):
         return torch.zeros_like(x)
     dev = _native.require_device(x)
     xf = _common.contiguous(x)
-    w = weight.to(device=dev, dtype=x.dtype).contiguous()
-    b = bias.to(device=dev, dtype=x.dtype).contiguous()
+    w = _common.as_param(weight, dev, x.dtype)
+    b = _common.as_param(bias, dev, x.dtype)
     y = torch.empty_like(xf)
     _native.check(
         _native.lib().motif_polynorm(
