@@ -33,11 +33,16 @@ bool mfma_q_bf16_ok(const SdpaArgs& a, int D, int gs);
 // softmax handles, and qpair 1 (4-bit caches; the default) or 2 (both).
 bool qpair_bf16_ok(const SdpaArgs& a, int D, int gs, int bits);
 
-// Packed cache (fp16 scales, head dim 128), a verify slab of 17..64 virtual
-// heads per KV head: tiles dequantised once per workgroup into LDS
-// (sdpa_qslab.hip); ncb column blocks of 16 heads (2 or 4), 4 or 8 waves.
-int launch_sdpa_qslab(const SdpaArgs& a, int bits, int gs, int ncb, int waves, int nblocks,
-                      hipStream_t s);
+// Packed cache (head dim 128), a verify slab of 17..64 virtual heads per KV
+// head: tiles dequantised once per workgroup into LDS (sdpa_qslab.hip); ncb
+// column blocks of 16 heads (2 or 4), 4 or 8 waves (bf16: 8, tuning qslab_ws).
+int launch_sdpa_qslab(const SdpaArgs& a, bool bf16, int bits, int gs, int ncb, int waves,
+                      int nblocks, hipStream_t st);
+
+// Prompt chunks over the packed cache (sdpa_qprefill.hip); fp16 or bf16 q,
+// scales and y, plan_prefill's waves and column blocks.
+int launch_sdpa_qprefill(const SdpaArgs& a, bool bf16, int bits, int waves, int ncb, int nblocks,
+                         hipStream_t st);
 
 // Prompt chunks over the packed cache (sdpa_qprefill.hip); fp16 or bf16 q,
 // scales and y, plan_prefill's waves and column blocks.

@@ -281,7 +281,12 @@ static int sdpa_q_run(const char* name, const void* q, const uint32_t* kd, const
   // dequantised once per workgroup into LDS and shared by its waves (with
   // producer and consumer waves: 5-row slab over 32768 rows, q8 33.0 against
   // 49.0 us in head chunks, q4 35.3 against 43.6 us).
-  if (dtype == MOTIF_F16 && D == 128 && tuning().mfma && tuning().qslab >= (bits == 8 ? 1 : 2) &&
+  const bool scan_ok = kv_cap % 4 == 0 && aligned(ks, 8) && aligned(kb, 8) && aligned(v1s, 8) &&
+                       aligned(v1b, 8) && aligned(v2s, 8) && aligned(v2b, 8);  // scan_scales
+  const bool bf16_slab = dtype == MOTIF_BF16 && scan_ok && tuning().qslab_ws &&
+                         tuning().waves_per_wg != 4;
+  if ((dtype == MOTIF_F16 || bf16_slab) && D == 128 && tuning().mfma &&
+      tuning().qslab >= (bits == 8 ? 1 : 2) &&
       a.GV >= kQSlabMinHeads && a.GV <= kQSlabMaxHeads && kv_len <= kMfmaMaxRows &&
       tile_softmax_scale_ok(a.qscale) &&
       aligned(q, 16) && aligned(y, 16) && aligned(kd, bits == 8 ? 16 : 8) &&
@@ -299,7 +304,7 @@ static int sdpa_q_run(const char* name, const void* q, const uint32_t* kd, const
     a.fused_merge = 0;
     rc = check_partials(name, a, false);
     if (rc != MOTIF_OK) return rc;
-    rc = launch_sdpa_qslab(a, bits, gs, qp.ncb, qp.waves,
+    rc = launch_sdpa_qslab(a, dtype == MOTIF_BF16, bits, gs, qp.ncb, qp.waves,
                            sdpa_grid_blocks(B * Hkv, qp.nchunk, qp.nsplit), s);
     return rc == MOTIF_OK ? sdpa_merge(a, dtype, D, s) : rc;
   }
@@ -309,11 +314,9 @@ static int sdpa_q_run(const char* name, const void* q, const uint32_t* kd, const
   // kernel / here: 382 / 120 us, error against 64 bits 8.7e-4 / 6.6e-4.
   if ((dtype == MOTIF_F16 || dtype == MOTIF_BF16) && D == 128 && tuning().mfma &&
       tuning().qslab >= (bits == 8 ? 1 : 2) && a.GV > kQSlabMaxHeads &&
-      use_shared_tiles(a.GV, kv_len) && kv_len <= kMfmaMaxRows && kv_cap % 4 == 0 &&
+      use_shared_tiles(a.GV, kv_len) && kv_len <= kMfmaMaxRows && scan_ok &&
       tile_softmax_scale_ok(a.qscale) && aligned(q, 16) && aligned(y, 16) &&
-      aligned(kd, bits) && aligned(v1d, bits) && aligned(v2d, bits) && aligned(ks, 8) &&
-      aligned(kb, 8) && aligned(v1s, 8) && aligned(v1b, 8) && aligned(v2s, 8) &&
-      aligned(v2b, 8)) {
+      aligned(kd, bits) && aligned(v1d, bits) && aligned(v2d, bits)) {
     const PrefillPlan pp = plan_prefill(B, Hq, Hkv, S_q, kv_len, D);
     a.counters = nullptr;
     a.part_o = a.part_ml = nullptr;

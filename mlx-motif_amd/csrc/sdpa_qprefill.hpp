@@ -26,35 +26,6 @@
 
 namespace motif {
 
-// Exponent of a positive float (-127 for zero and subnormals).
-__device__ inline int float_exp(float x) {
-  return (int)((__builtin_bit_cast(uint32_t, x) >> 23) & 0xFFu) - 127;
-}
-// e with |s * u + b| * 2^-e < 2^15 for every code u <= 255, given m = max(|s|,
-// |b| / 256): |s| * 255 + |b| < 2^9 m < 2^(exp(m) + 10).  fp16 rows are
-// scaled down only (almost always e = 0, their scales as stored).
-template <typename E>
-__device__ inline int value_exp(float m) {
-  const int e = float_exp(m) - 5;
-  return std::is_same<E, bf16_t>::value ? e : max(e, 0);
-}
-// qscale * 2^e, kept finite and above zero (0 * inf at a masked row).
-__device__ inline float scaled_qscale(float qscale, int e) {
-  return fminf(fmaxf(ldexpf(qscale, e), 1.1754943508222875e-38f), 3.4028234663852886e38f);
-}
-
-// A scale or bias as stored (16 bits of E), times 2^-e, in both halves of an
-// fp16 pair.  h2: 2^-e in both halves (fp16 rows, 0 <= e).
-template <typename E>
-__device__ inline half2_t scale_pair(uint32_t bits, int e, half2_t h2) {
-  if constexpr (std::is_same<E, bf16_t>::value) {
-    const _Float16 v = (_Float16)ldexpf(__builtin_bit_cast(float, bits << 16), -e);
-    return half2_t{v, v};
-  } else {
-    return as_h2((bits & 0xFFFFu) | (bits << 16)) * h2;
-  }
-}
-
 // 8 codes as fp16 s * u + b (one rounding each): two codes become 1024 + u in
 // the halves of one word, a packed subtract leaves u exactly, a packed fma
 // gives the value.
@@ -165,8 +136,7 @@ sdpa_qprefill_kernel(SdpaArgs a) {
   load(P, 0);
 
   // Powers of two of K, V1 and V2 from the scales and biases of this split's
-  // rows, four halves per load (whole 4-row groups: kv_cap % 4 == 0; halves
-  // of rows past r_end are dropped).
+  // rows.
   // Stage st, tensor t: 32 rows x 256 bytes, 16-byte chunk c of row r at byte
   // r * 256 + (c ^ (r % 16)) * 16; the split partials are staged there at the end.
   constexpr int TB = TR * D * 2;
@@ -175,30 +145,8 @@ sdpa_qprefill_kernel(SdpaArgs a) {
   __shared__ float wmax[3][NW];
   int ex[3];
   {
-    float m[3] = {0.f, 0.f, 0.f};
-    const unsigned s4bytes = (unsigned)((r_end + 3) & ~3) << (lg + 1);
-    const int per_tile = 8 << lg;  // 8-byte words of a tile's rows
-    for (int i = tid; i < ntiles * per_tile; i += NW * 64) {
-      const int tile = i >> (3 + lg);
-      const int h0 = 4 * (i & (per_tile - 1));
-      const int row0 = (tile * ns + split) * TR;
-      const unsigned off = (((unsigned)row0 << lg) + (unsigned)h0) * 2u;
-      const void* sp[3] = {a.ks, a.v1s, a.v2s};
-      const void* bp[3] = {a.kb, a.v1b, a.v2b};
-#pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        const uint2 s = bload2<0>(uniform_stream_rsrc(head_scales(sp[t]), s4bytes), off);
-        const uint2 b = bload2<0>(uniform_stream_rsrc(head_scales(bp[t]), s4bytes), off);
-        const uint32_t sw[2] = {s.x, s.y}, bw[2] = {b.x, b.y};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint16_t sh = (uint16_t)(sw[j / 2] >> (16 * (j % 2)));
-          const uint16_t bh = (uint16_t)(bw[j / 2] >> (16 * (j % 2)));
-          const float v = fmaxf(fabsf(Elem<E>::to_f32(sh)), fabsf(Elem<E>::to_f32(bh)) * 0x1p-8f);
-          m[t] = row0 + ((h0 + j) >> lg) < r_end ? fmaxf(m[t], v) : m[t];
-        }
-      }
-    }
+    float m[3];
+    scan_scales<E>(a, hrow0, lg, split * TR, ns * TR, ntiles, r_end, tid, NW * 64, m);
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
       const float x = group_max<64>(m[t]);
@@ -227,25 +175,7 @@ sdpa_qprefill_kernel(SdpaArgs a) {
     for (int s = 0; s < 4; ++s)
       w[s] = col_ok[cb] ? *reinterpret_cast<const uint4*>(qp + 32 * s) : make_uint4(0, 0, 0, 0);
     int qe = 0;
-    if constexpr (kBf16) {
-      float mx = 0.f;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const uint32_t x[4] = {w[s].x, w[s].y, w[s].z, w[s].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          mx = fmaxf(mx, fmaxf(fabsf(pair_lo_f32<E>(x[i])), fabsf(pair_hi_f32<E>(x[i]))));
-      }
-      qe = float_exp(rows4_max(mx)) - 14;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        uint32_t x[4] = {w[s].x, w[s].y, w[s].z, w[s].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          x[i] = f16_pair(ldexpf(pair_lo_f32<E>(x[i]), -qe), ldexpf(pair_hi_f32<E>(x[i]), -qe));
-        w[s] = make_uint4(x[0], x[1], x[2], x[3]);
-      }
-    }
+    if constexpr (kBf16) qe = q_row_f16(w);
 #pragma unroll
     for (int s = 0; s < 4; ++s) qb[cb][s] = __builtin_bit_cast(V8, w[s]);
     qsc[cb] = scaled_qscale(a.qscale, ex[0] + qe);
