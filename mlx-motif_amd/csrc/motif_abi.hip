@@ -238,19 +238,37 @@ GdaPrefillPlan plan_gda_prefill(int B, int Hkv, int G_origin, int G_noise, int S
   if (tuning().rows_per_split > 0) {
     const int rps = (int)round_up((size_t)tuning().rows_per_split, kPrefillTileRowsHost);
     nsplit = (rows + rps - 1) / rps;
-  } else if (units < cus / 2) {
-    // Workgroups hold one CU each (the LDS ring).  Few query blocks: as many
-    // splits (tiles dealt round robin) as keep the workgroups within one
-    // round, at least 4 tiles each.
-    nsplit = (int)std::min<long>(std::max<long>(cus / units, 1), std::max(1, tiles / 4));
+  } else if (units < cus) {
+    // Workgroups hold one CU each (the LDS ring): as many splits (tiles dealt
+    // round robin) as keep them within one round, at least 4 tiles each, or
+    // two rounds with at least 32 tiles each (each workgroup's prologue,
+    // partials and the merge launch cost more than a round's idle CUs on
+    // short ranges).  A 512-row chunk of 32 + 8 heads over 8 KV heads at
+    // offset 3204 (160 blocks): 1 / 2 / 3 / 4 splits 158 / 180 / 141 / 165 us;
+    // at offset 0: 1 / 2 splits 42 / 67 us.
+    nsplit = fill_splits(units, cus, tiles / 32);
+    nsplit = std::min(nsplit, std::max(1, tiles / 4));
   } else {
-    // Enough blocks for most CUs: split only while the workgroups fit two
-    // rounds and every split keeps at least 32 tiles (each workgroup's
-    // prologue, partials and the merge launch cost more than a round's idle
-    // CUs on short ranges).  A 512-row chunk of 32 + 8 heads over 8 KV heads
-    // at offset 3204 (160 blocks): 1 / 2 / 3 / 4 splits 158 / 180 / 141 /
-    // 165 us; at offset 0: 1 / 2 splits 42 / 67 us.
-    for (int k = 2; units * k <= 2L * cus && tiles / k >= 32; ++k) nsplit = k;
+    // More blocks than CUs: whole rounds unsplit, and the last, partly filled
+    // round's blocks split to fill it (fp32 partials of those alone), where
+    // every split keeps 16 tiles and every block sees at least 64 (in a first
+    // chunk's blocks the causal limit already spreads their lengths).
+    // 2048 rows at offset 6150, fp16, 320 blocks, one layer's pass: 649 us in
+    // two rounds, 479 us with the noise pass's 64 blocks in 4 splits.
+    const long bh = (long)B * Hkv;
+    const int nqb = p.nqb_origin + p.nqb_noise;
+    const int full = (int)(units / cus * cus / bh);
+    if (full > 0 && full < nqb && kv_len - S >= 64 * kPrefillTileRowsHost) {
+      const int k = std::min(fill_splits((nqb - full) * bh, cus, tiles / 16), tiles / 16);
+      if (k > 1) {
+        nsplit = k;
+        p.nq_full = full;
+        p.tail_o0 = std::min(full, p.nqb_origin) * cols;
+        if (p.tail_o0 > G_origin * S) p.tail_o0 = G_origin * S;
+        p.tail_n0 = std::max(full - p.nqb_origin, 0) * cols;
+        p.tail_rows = G_origin * S - p.tail_o0 + G_noise * S - p.tail_n0;
+      }
+    }
   }
   if (nsplit > kMaxSplits) nsplit = kMaxSplits;
   int rps = (rows + nsplit - 1) / nsplit;
@@ -258,7 +276,8 @@ GdaPrefillPlan plan_gda_prefill(int B, int Hkv, int G_origin, int G_noise, int S
   p.rows_per_split = rps;
   p.nsplit = (rows + rps - 1) / rps;
   if (p.nsplit > 1) {
-    const size_t vrows = (size_t)B * Hkv * (G_origin + G_noise) * S;
+    const size_t vrows =
+        (size_t)B * Hkv * (p.nq_full > 0 ? p.tail_rows : (G_origin + G_noise) * S);
     p.workspace_bytes = round_up(vrows * sizeof(unsigned), 256) +
                         round_up(vrows * p.nsplit * 2 * 128 * sizeof(float), 256) +
                         round_up(vrows * p.nsplit * 2 * sizeof(float), 256);

@@ -1136,7 +1136,14 @@ int motif_gda_prefill_proj_scaled(const void* q_proj, const void* k_proj, const 
   const int kv_len = offset + S;
   const int Hq_o = q_groups * gr;
   const int G_o = Hq_o / k_groups, G_n = q_groups / k_groups;
-  const GdaPrefillPlan pp = plan_gda_prefill(B, k_groups, G_o, G_n, S, kv_len);
+  GdaPrefillPlan pp = plan_gda_prefill(B, k_groups, G_o, G_n, S, kv_len);
+  // (a split tail is an option: without its workspace every block runs whole)
+  if (pp.nq_full > 0 && (workspace == nullptr || workspace_bytes < pp.workspace_bytes)) {
+    pp.nq_full = 0;
+    pp.nsplit = 1;
+  }
+  const long part_rows = pp.nq_full > 0 ? (long)B * k_groups * pp.tail_rows
+                                        : (long)B * (Hq_o + q_groups) * S;
   SdpaArgs a{};
   a.q = y_origin; a.q2 = y_noise; a.q_stride = 2 * D;  // q roped into the rows of y, below
   a.k = k1; a.k2 = k2; a.v1 = v1; a.v2 = v2;
@@ -1153,12 +1160,17 @@ int motif_gda_prefill_proj_scaled(const void* q_proj, const void* k_proj, const 
   a.tiles_rr = 1;
   a.y2_row0 = (long)B * Hq_o * S;
   if (pp.nsplit > 1) {
-    const int rc = carve_split_ws(name, a, workspace, workspace_bytes,
-                                  (size_t)B * (Hq_o + q_groups) * S, pp.nsplit, D, 0);
+    const int rc = carve_split_ws(name, a, workspace, workspace_bytes, (size_t)part_rows,
+                                  pp.nsplit, D, 0);
     if (rc != MOTIF_OK) return rc;
   }
-  a.part_f16 =
-      use_part_f16((long)B * (Hq_o + q_groups) * S, pp.nsplit, dtype == MOTIF_F16) ? 1 : 0;
+  a.nq_full = pp.nq_full;
+  a.blocks_full = pp.nq_full > 0 ? sdpa_grid_blocks(B * k_groups, pp.nq_full, 1) : 0;
+  a.tail_rows = pp.tail_rows;
+  a.tail_o0 = pp.tail_o0;
+  a.tail_n0 = pp.tail_n0;
+  // (the blocks of a split tail keep fp32 partials, the precision of the others)
+  a.part_f16 = pp.nq_full == 0 && use_part_f16(part_rows, pp.nsplit, dtype == MOTIF_F16) ? 1 : 0;
   int rc = check_partials(name, a, false);
   if (rc != MOTIF_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
@@ -1175,7 +1187,7 @@ int motif_gda_prefill_proj_scaled(const void* q_proj, const void* k_proj, const 
                           q_groups, gr, k_groups, 1, D, kv_cap, offset, offset, theta,
                           position_scale, origin_first, 2 * D, s);
   if (rc != MOTIF_OK) return rc;
-  const int nblocks = sdpa_grid_blocks(B * k_groups, a.nchunk, pp.nsplit);
+  const int nblocks = a.blocks_full + sdpa_grid_blocks(B * k_groups, a.nchunk - a.nq_full, pp.nsplit);
   rc = dtype == MOTIF_F16 ? launch_sdpa_prefill_f16(a, pp.waves, pp.ncb, nblocks, s)
                           : launch_sdpa_prefill_bf16(a, pp.waves, pp.ncb, nblocks, s);
   if (rc != MOTIF_OK || pp.nsplit == 1) return rc;
@@ -1249,7 +1261,7 @@ int motif_plan_selfcheck(void) {
     clear_error();
   }
   const int heads[][2] = {{32, 8}, {40, 8}, {8, 8}, {4, 4}, {16, 4}, {64, 8}, {128, 8}};
-  const int rows_q[] = {1, 2, 5, 17, 37, 128, 512};
+  const int rows_q[] = {1, 2, 5, 17, 37, 128, 512, 1700, 2048};
   const int lens[] = {0, 1, 15, 16, 17, 300, 1024, 2047, 2048, 3204, 4096, 4097, 16000, 32768,
                       131072};
   constexpr int D = 128;
@@ -1315,7 +1327,28 @@ int motif_plan_selfcheck(void) {
             if (q_groups % Hkv == 0) {
               const int G_o = q_groups * gr / Hkv, G_n = q_groups / Hkv;
               const GdaPrefillPlan gp = plan_gda_prefill(B, Hkv, G_o, G_n, S_q, kv_len);
-              const size_t gv_rows = (size_t)B * (q_groups * gr + q_groups) * S_q;
+              // a split tail: every split row has its own partial row, which
+              // the merge maps back to the row's place in y or y2
+              if (gp.nq_full > 0) {
+                SdpaArgs t{};
+                t.GV = G_o * S_q; t.G2 = G_n; t.S_q = S_q;
+                t.tail_rows = gp.tail_rows; t.tail_o0 = gp.tail_o0; t.tail_n0 = gp.tail_n0;
+                t.y2_row0 = (long)B * Hkv * t.GV;
+                long next = 0;
+                for (int unit = 0; unit < B * Hkv; ++unit)
+                  for (int noise = 0; noise < 2; ++noise) {
+                    const int heads = noise ? G_n * S_q : t.GV;
+                    for (int vh = noise ? t.tail_n0 : t.tail_o0; vh < heads; ++vh, ++next)
+                      if (TailRows::part_row(t, unit, noise != 0, vh) != next ||
+                          TailRows::out_row(t, next) !=
+                              (noise ? t.y2_row0 : 0) + (long)unit * heads + vh)
+                        return fail("split tail rows", B, Hq, Hkv, S_q, kv_len, gp.nsplit);
+                  }
+                if (next != (long)B * Hkv * gp.tail_rows)
+                  return fail("split tail row count", B, Hq, Hkv, S_q, kv_len, gp.nsplit);
+              }
+              const size_t gv_rows = gp.nq_full > 0 ? (size_t)B * Hkv * gp.tail_rows
+                                                    : (size_t)B * (q_groups * gr + q_groups) * S_q;
               if ((rc = check_plan("gda prefill plan", gv_rows, gp.nsplit, gp.workspace_bytes, B,
                                    Hq, Hkv, S_q, kv_len, 0)) != MOTIF_OK)
                 return rc;

@@ -714,10 +714,11 @@ __device__ inline void merge_rows(const SdpaArgs& a, long vrow, int lane) {
   for (int k = 0; k < CPL; ++k) {
     const int c = lane + 64 * k;
     if (c >= C4) continue;
-    if (a.y2 != nullptr && vrow >= a.y2_row0)  // second output (fused prefill's noise pass)
-      store_y4_to<T, D>(a.y2, (vrow - a.y2_row0) * 2 * D + c * 4, acc[k], L);
+    const long yrow = a.nq_full > 0 ? TailRows::out_row(a, vrow) : vrow;
+    if (a.y2 != nullptr && yrow >= a.y2_row0)  // second output (fused prefill's noise pass)
+      store_y4_to<T, D>(a.y2, (yrow - a.y2_row0) * 2 * D + c * 4, acc[k], L);
     else
-      store_y4<T, D>(a, vrow * 2 * D + c * 4, acc[k], L);
+      store_y4<T, D>(a, yrow * 2 * D + c * 4, acc[k], L);
   }
 }
 
@@ -815,14 +816,15 @@ __global__ void __launch_bounds__(256) sdpa_merge_rows16_kernel(SdpaArgs a, long
 // The merge launch takes the row-per-wave kernel for this call (many partial
 // rows, or fp16 partials, which only that kernel reads).
 inline bool merge_uses_rows_kernel(const SdpaArgs& a) {
-  return a.part_f16 || ((long)a.B * a.Hq * a.S_q >= kMergeRowsMin && tuning().merge_rows);
+  return a.part_f16 || a.nq_full > 0 || ((long)a.B * a.Hq * a.S_q >= kMergeRowsMin && tuning().merge_rows);
 }
 
 template <typename T, int D>
 int launch_sdpa_merge_d(const SdpaArgs& a, hipStream_t s) {
   constexpr int C4 = 2 * D / 4;
   constexpr int NSL = C4 / (C4 < 16 ? C4 : 16);
-  const long rows = (long)a.B * a.Hq * a.S_q;
+  const long rows =
+      a.nq_full > 0 ? (long)a.B * a.Hkv * a.tail_rows : (long)a.B * a.Hq * a.S_q;
   if constexpr (64 % (2 * D / 8) == 0) {
     // fp16 partials: 16-byte loads, whole rows per wave (prefill chunk of
     // 512 rows over 3716: 69.6 against 71.5-75.8 us per call with the

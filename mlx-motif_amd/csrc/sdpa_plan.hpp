@@ -93,10 +93,33 @@ struct SdpaArgs {
   // noise pass (G2 heads: q2 x k2, output y2, whose split partials start at
   // row y2_row0).
   int q_stride;
+  // Query blocks [0, nq_full) of every (b, KV head) unsplit, the others in
+  // nsplit splits (0: every block in nsplit).  The grid's first blocks_full
+  // workgroups are the unsplit ones.  Partial rows are then the split blocks'
+  // only, tail_rows per (b, KV head): the origin pass's virtual heads from
+  // tail_o0 on, then the noise pass's from tail_n0 on (TailRows).
+  int nq_full, blocks_full;
+  int tail_rows, tail_o0, tail_n0;
   void* y2;
   long y2_row0;
   int nqb_origin;
   int G2;  // noise heads per KV head (the prefill chunk and the fused decode step)
+};
+
+// Partial rows of a launch whose last query blocks alone are split.
+struct TailRows {
+  // Partial row of virtual head vh of a pass of (b, KV head) unit.
+  __host__ __device__ static long part_row(const SdpaArgs& a, int unit, bool noise, int vh) {
+    return (long)unit * a.tail_rows + (noise ? a.GV - a.tail_o0 + vh - a.tail_n0 : vh - a.tail_o0);
+  }
+  // Output row of partial row r: a row of y, or y2_row0 plus a row of y2.
+  __host__ __device__ static long out_row(const SdpaArgs& a, long r) {
+    const long unit = r / a.tail_rows;
+    const int j = (int)(r % a.tail_rows);
+    const int n_o = a.GV - a.tail_o0;  // the origin pass's split heads
+    return j < n_o ? unit * a.GV + a.tail_o0 + j
+                   : a.y2_row0 + unit * ((long)a.G2 * a.S_q) + a.tail_n0 + (j - n_o);
+  }
 };
 
 struct SdpaPlan {
@@ -165,6 +188,8 @@ struct GdaPrefillPlan {
   int ncb;  // column blocks of 16 virtual heads per wave (1 or 2)
   int nqb_origin, nqb_noise;
   int nsplit, rows_per_split;
+  int nq_full;  // query blocks left unsplit (SdpaArgs::nq_full), 0: all alike
+  int tail_rows, tail_o0, tail_n0;
   size_t workspace_bytes;  // counters + partials, 0 when nsplit == 1
 };
 GdaPrefillPlan plan_gda_prefill(int B, int Hkv, int G_origin, int G_noise, int S, int kv_len);

@@ -91,6 +91,29 @@ __device__ inline bool prefill_block_coords(const SdpaArgs& a, int bid, int& qbl
   return true;
 }
 
+// The same where only the query blocks from nq_full on are split: ns is the
+// block's own split count.
+__device__ inline bool prefill_tail_coords(const SdpaArgs& a, int bid, int& qblk, int& unit,
+                                           int& split, int& ns) {
+  int nq = a.nchunk, first = 0;
+  ns = a.nsplit;
+  if (a.nq_full > 0) {
+    const bool full = bid < a.blocks_full;
+    first = full ? 0 : a.nq_full;
+    nq = full ? a.nq_full : a.nchunk - a.nq_full;
+    ns = full ? 1 : ns;
+    bid -= full ? 0 : a.blocks_full;
+  }
+  const int bh = a.B * a.Hkv;
+  const int slot = bid >> 3;
+  qblk = first + slot % nq;
+  const int g = (slot / nq) * 8 + (bid & 7);
+  if (g >= bh * ns) return false;
+  split = g / bh;
+  unit = g % bh;
+  return true;
+}
+
 // One column's online-softmax state over 32-row fp16/bf16 K/V tiles held in
 // LDS with 16-byte chunk c of row r at byte r * 256 + (c ^ (r % 16)) * 16:
 // S^T = K Q^T (16x16x32 MFMA, two 16-row halves), scores in log2 units with
@@ -432,8 +455,8 @@ sdpa_prefill_kernel(SdpaArgs a) {
   const int col = lane & 15;
   const int blk = lane >> 4;
 
-  int qblk, unit, split;
-  if (!prefill_block_coords(a, blockIdx.x, qblk, unit, split)) return;  // grid padding
+  int qblk, unit, split, ns;
+  if (!prefill_tail_coords(a, blockIdx.x, qblk, unit, split, ns)) return;  // grid padding
   // A layer's chunk (gda_prefill_proj) has query blocks of two passes: the
   // origin heads over k, then from block nqb_origin on the noise heads over
   // k2, both over v1 / v2.
@@ -465,7 +488,6 @@ sdpa_prefill_kernel(SdpaArgs a) {
   // causal limit) or in contiguous ranges of rows_per_split rows (tile
   // i of split s is tile s * tps + i).  Rows at or past r_end = max_lim are
   // masked.
-  const int ns = a.nsplit;
   const int r_end = max_lim;
   const int tps = a.rows_per_split / TR;  // tiles per contiguous range
   const int tstride = a.tiles_rr ? ns : 1;
@@ -595,8 +617,10 @@ sdpa_prefill_kernel(SdpaArgs a) {
   }
 
   // acc[j][r] of lane (col, blk) is channel 32*blk + 4*j + r of column col.
-  const long prow0 = (noise ? a.y2_row0 : 0) + qrow0;  // its split partials' row
-  if (a.nsplit > 1) {
+  // its split partials' row
+  const long prow0 = a.nq_full > 0 ? TailRows::part_row(a, unit, noise, 0)
+                                   : (noise ? a.y2_row0 : 0) + qrow0;
+  if (ns > 1) {
     // Partials through the ring, once every wave is done with it.
     static_assert(NW * kStageWaveBytes <= (int)sizeof(ring), "staging fits the ring");
     __syncthreads();
@@ -605,7 +629,7 @@ sdpa_prefill_kernel(SdpaArgs a) {
     for (int cb = 0; cb < NCB; ++cb) {
       const int c0 = vh[cb] - col;  // the block's first virtual head
       store_partials_staged<T>(st_acc[cb], lds, a.part_o, a.part_ml, prow0 + c0,
-                               min(16, GV - c0), a.nsplit, split, col, blk, a.part_f16);
+                               min(16, GV - c0), ns, split, col, blk, a.part_f16);
     }
     return;
   }
@@ -613,7 +637,7 @@ sdpa_prefill_kernel(SdpaArgs a) {
   for (int cb = 0; cb < NCB; ++cb)
     if (col_ok[cb])
       st_acc[cb].store_to(noise ? a.y2 : a.y, qrow0 + vh[cb], a.part_o, a.part_ml, prow0 + vh[cb],
-                          a.nsplit, split, blk, a.part_f16);
+                          ns, split, blk, a.part_f16);
 }
 
 template <typename T>
