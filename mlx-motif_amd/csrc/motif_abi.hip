@@ -240,25 +240,27 @@ GdaPrefillPlan plan_gda_prefill(int B, int Hkv, int G_origin, int G_noise, int S
     nsplit = (rows + rps - 1) / rps;
   } else if (units < cus) {
     // Workgroups hold one CU each (the LDS ring): as many splits (tiles dealt
-    // round robin) as keep them within one round, at least 4 tiles each, or
+    // round robin) as keep them within one round, at least 8 tiles each (333
+    // rows at offset 0, 11 tiles: 1 / 2 splits 30 / 37 us), or
     // two rounds with at least 32 tiles each (each workgroup's prologue,
     // partials and the merge launch cost more than a round's idle CUs on
     // short ranges).  A 512-row chunk of 32 + 8 heads over 8 KV heads at
     // offset 3204 (160 blocks): 1 / 2 / 3 / 4 splits 158 / 180 / 141 / 165 us;
     // at offset 0: 1 / 2 splits 42 / 67 us.
     nsplit = fill_splits(units, cus, tiles / 32);
-    nsplit = std::min(nsplit, std::max(1, tiles / 4));
+    nsplit = std::min(nsplit, std::max(1, tiles / 8));
   } else {
     // More blocks than CUs: whole rounds unsplit, and the last, partly filled
     // round's blocks split to fill it (fp32 partials of those alone), where
-    // every split keeps 16 tiles and every block sees at least 64 (in a first
-    // chunk's blocks the causal limit already spreads their lengths).
+    // every split keeps 16 tiles.  With fewer rows before the chunk the causal
+    // limit spreads the blocks' lengths so far that longest first fills the
+    // rounds as well (prefill_order).
     // 2048 rows at offset 6150, fp16, 320 blocks, one layer's pass: 649 us in
     // two rounds, 479 us with the noise pass's 64 blocks in 4 splits.
     const long bh = (long)B * Hkv;
     const int nqb = p.nqb_origin + p.nqb_noise;
     const int full = (int)(units / cus * cus / bh);
-    if (full > 0 && full < nqb && kv_len - S >= 64 * kPrefillTileRowsHost) {
+    if (full > 0 && full < nqb && 8L * (kv_len - S) >= 5L * S) {
       const int k = std::min(fill_splits((nqb - full) * bh, cus, tiles / 16), tiles / 16);
       if (k > 1) {
         nsplit = k;

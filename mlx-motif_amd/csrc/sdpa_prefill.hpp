@@ -23,6 +23,8 @@
 // streams only the rows its columns can see.
 #pragma once
 
+#include <algorithm>
+
 #include "sdpa_mfma_q.hpp"
 
 namespace motif {
@@ -91,10 +93,40 @@ __device__ inline bool prefill_block_coords(const SdpaArgs& a, int bid, int& qbl
   return true;
 }
 
+// Order in which the query blocks of a (b, KV head, split) are started (n = 0:
+// as they are numbered).  Under the causal limit a block's tiles grow with its
+// last query row; where more workgroups than CUs are launched, the longest go
+// first, so that the last to start are the shortest.
+constexpr int kPrefillOrderMax = 252;
+struct PrefillOrder {
+  int n;
+  uint8_t blk[kPrefillOrderMax];
+};
+inline PrefillOrder prefill_order(const SdpaArgs& a, int cols, int nblocks) {
+  PrefillOrder o;
+  o.n = 0;
+  if (!a.causal || a.nchunk < 2 || a.nchunk > kPrefillOrderMax || nblocks <= device_cu_count())
+    return o;
+  int last[kPrefillOrderMax];  // last query row among the block's virtual heads
+  for (int b = 0; b < a.nchunk; ++b) {
+    const bool noise = b >= a.nqb_origin;
+    const int v0 = (noise ? b - a.nqb_origin : b) * cols;
+    const int n = std::min(cols, (noise ? a.G2 * a.S_q : a.GV) - v0);
+    last[b] = v0 % a.S_q + n > a.S_q ? a.S_q - 1 : v0 % a.S_q + n - 1;
+    o.blk[b] = (uint8_t)b;
+  }
+  // (the unsplit blocks and a split tail stay in their own parts of the grid)
+  auto longer = [&](uint8_t x, uint8_t y) { return last[x] > last[y]; };
+  std::stable_sort(o.blk, o.blk + a.nq_full, longer);
+  std::stable_sort(o.blk + a.nq_full, o.blk + a.nchunk, longer);
+  o.n = a.nchunk;
+  return o;
+}
+
 // The same where only the query blocks from nq_full on are split: ns is the
 // block's own split count.
-__device__ inline bool prefill_tail_coords(const SdpaArgs& a, int bid, int& qblk, int& unit,
-                                           int& split, int& ns) {
+__device__ inline bool prefill_tail_coords(const SdpaArgs& a, const PrefillOrder& order, int bid,
+                                           int& qblk, int& unit, int& split, int& ns) {
   int nq = a.nchunk, first = 0;
   ns = a.nsplit;
   if (a.nq_full > 0) {
@@ -107,6 +139,7 @@ __device__ inline bool prefill_tail_coords(const SdpaArgs& a, int bid, int& qblk
   const int bh = a.B * a.Hkv;
   const int slot = bid >> 3;
   qblk = first + slot % nq;
+  if (order.n > 0) qblk = order.blk[qblk];
   const int g = (slot / nq) * 8 + (bid & 7);
   if (g >= bh * ns) return false;
   split = g / bh;
@@ -445,7 +478,7 @@ __device__ inline __amdgpu_buffer_rsrc_t uniform_stream_rsrc(const void* base, u
 // read from LDS feeds two blocks' MFMAs, half the LDS reads per head).
 template <typename T, int NW, int NS = kPrefillStages, int NCB = 1>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 2 : 1)))
-sdpa_prefill_kernel(SdpaArgs a) {
+sdpa_prefill_kernel(SdpaArgs a, PrefillOrder order) {
   using Op = MfmaOp<T>;
   using V8 = typename Op::V8;
   constexpr int D = 128;
@@ -456,7 +489,7 @@ sdpa_prefill_kernel(SdpaArgs a) {
   const int blk = lane >> 4;
 
   int qblk, unit, split, ns;
-  if (!prefill_tail_coords(a, blockIdx.x, qblk, unit, split, ns)) return;  // grid padding
+  if (!prefill_tail_coords(a, order, blockIdx.x, qblk, unit, split, ns)) return;  // grid padding
   // A layer's chunk (gda_prefill_proj) has query blocks of two passes: the
   // origin heads over k, then from block nqb_origin on the noise heads over
   // k2, both over v1 / v2.
@@ -643,13 +676,14 @@ sdpa_prefill_kernel(SdpaArgs a) {
 template <typename T>
 inline int launch_prefill_kernel_16(const SdpaArgs& a, int waves, int ncb, int nblocks,
                                    hipStream_t st) {
+  const PrefillOrder order = prefill_order(a, waves * 16 * (waves == 8 ? ncb : 1), nblocks);
   if (waves == 8 && ncb == 2) {
     hipLaunchKernelGGL((sdpa_prefill_kernel<T, 8, kPrefillStages, 2>), dim3(nblocks), dim3(512),
-                       0, st, a);
+                       0, st, a, order);
   } else if (waves == 8) {
-    hipLaunchKernelGGL((sdpa_prefill_kernel<T, 8>), dim3(nblocks), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((sdpa_prefill_kernel<T, 8>), dim3(nblocks), dim3(512), 0, st, a, order);
   } else {
-    hipLaunchKernelGGL((sdpa_prefill_kernel<T, 4>), dim3(nblocks), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((sdpa_prefill_kernel<T, 4>), dim3(nblocks), dim3(256), 0, st, a, order);
   }
   return check_launch("sdpa_dual_v_rows (prefill)");
 }
