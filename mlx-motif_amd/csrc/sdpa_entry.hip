@@ -363,6 +363,13 @@ static GdaDecodeLayout gda_decode_layout(int B, int Hkv, int G1, int G2, int kv_
   const bool short4 = kv_len <= kShortDecodeRows;
   L.plan = plan_sdpa(B, Hkv, Hkv, 1, kv_len, D, 1, short4 ? 4 : 0, short4 ? 1 : 0);
   L.plan_q = plan_sdpa(B, Hkv, Hkv, 1, kv_len, D, 1, kSdpaMfmaQWaves, kSdpaMfmaQWgsPerCu);
+  // Short contexts in one split: no partials and no merge launch.
+  if (kv_len <= kOneSplitRows && tuning().rows_per_split == 0 && tuning().min_wgs == 0) {
+    for (SdpaPlan* p : {&L.plan, &L.plan_q}) {
+      p->nsplit = 1;
+      p->rows_per_split = (kv_len + 127) / 128 * 128;
+    }
+  }
   const int ns = L.plan.nsplit > L.plan_q.nsplit ? L.plan.nsplit : L.plan_q.nsplit;
   const size_t prow = (size_t)B * Hkv * (G1 + G2);
   L.counter_bytes = round256(prow * sizeof(unsigned));

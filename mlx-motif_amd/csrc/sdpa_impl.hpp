@@ -379,19 +379,87 @@ __device__ void merge_splits(const SdpaArgs& a, long qrow0, int nvh) {
   }
 }
 
+// A fused decode step of one split: the workgroup holds every head of its KV
+// head, so it applies gda_decode_merge_kernel's epilogue itself (same
+// operations per element) and the merge launch is left out.  Wave w takes
+// origin heads w, w + NW, ...; a lane's four channels of the head's row and of
+// its noise head's.
+template <typename T, int D, int GC, int NW>
+__device__ void gda_direct_epilogue(const SdpaArgs& a, const float (&lds_o)[NW][GC][2 * D + kLdsPad],
+                                    const float (&lds_m)[NW][GC], const float (&lds_l)[NW][GC],
+                                    long bk) {
+  static_assert(2 * D == 256, "64 lanes x 4 channels");
+  const int lane = threadIdx.x & 63;
+  const int c = 4 * lane;
+  const float lam = *a.gda_lambda;
+  float wv[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) wv[e] = Elem<T>::load(a.gda_w, c + e);
+  // o / l of column g over the waves, rounded to T (o when l == 0)
+  auto column = [&](int g, float (&o)[4]) {
+    float M = kNegSentinel;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, lds_m[w][g]);
+    float L = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = fast_exp2(lds_m[w][g] - M);
+      L = fmaf(lds_l[w][g], f, L);
+      const float4 v = *reinterpret_cast<const float4*>(&lds_o[w][g][c]);
+      o[0] = fmaf(v.x, f, o[0]);
+      o[1] = fmaf(v.y, f, o[1]);
+      o[2] = fmaf(v.z, f, o[2]);
+      o[3] = fmaf(v.w, f, o[3]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = L == 0.f ? o[e] : o[e] / L;
+      o[e] = Elem<T>::to_f32(Elem<T>::from_f32(x));
+    }
+  };
+  for (int i = threadIdx.x >> 6; i < a.G; i += NW) {
+    float o[4], n[4], d[4];
+    column(i, o);
+    column(a.G + i / (a.G / a.G2), n);
+    float ssq = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      d[e] = o[e] - lam * n[e];
+      ssq = fmaf(d[e], d[e], ssq);
+    }
+    ssq = group_sum<64>(ssq);
+    const float rms_inv = rsqrtf(ssq / (float)(2 * D) + a.gda_eps);
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = d[e] * rms_inv * wv[e] * a.gda_scale;
+    *reinterpret_cast<uint2*>((uint16_t*)a.y + (bk * a.G + i) * 2 * D + c) = make_uint2(
+        (uint32_t)Elem<T>::from_f32(y[0]) | ((uint32_t)Elem<T>::from_f32(y[1]) << 16),
+        (uint32_t)Elem<T>::from_f32(y[2]) | ((uint32_t)Elem<T>::from_f32(y[3]) << 16));
+  }
+}
+
 // ------------------------------------------------- workgroup epilogue ---
 // Combine the NW waves' (m, l, o1, o2) staged in LDS (log2-domain running
 // max, sum and unnormalised accumulators per virtual head), then either
 // write y (single split) or publish this split's partial with 16-byte
 // write-through stores and, in the workgroup that arrives last for its
 // (b, KV head, chunk), merge all splits.  Called by every thread of the
-// workgroup after a barrier.  PARTIALS: always publish partials (also for a
-// single split) and leave the merge to a second launch.
+// workgroup after a barrier.  PARTIALS (the fused decode step): publish
+// partials and leave the merge to a second launch; one split of a 16-bit type
+// at D = 128 finishes here (gda_direct_epilogue).
 template <typename T, int D, int GC, int NW, bool PARTIALS = false, bool FUSED_MERGE = true>
 __device__ void wg_epilogue(const SdpaArgs& a, const float (&lds_o)[NW][GC][2 * D + kLdsPad],
                             const float (&lds_m)[NW][GC], const float (&lds_l)[NW][GC],
                             long qrow0, int nvh, int split, int unit) {
   constexpr int C4 = 2 * D / 4;
+  if constexpr (PARTIALS && 2 * D == 256 && Elem<T>::kBytes == 2) {
+    if (a.nsplit == 1) {
+      gda_direct_epilogue<T, D, GC, NW>(a, lds_o, lds_m, lds_l, qrow0 / (a.G + a.G2));
+      return;
+    }
+  }
   const bool single = !PARTIALS && a.nsplit == 1;
   const int ns = a.nsplit;
   // (single split: no workspace, empty resources that are never used)

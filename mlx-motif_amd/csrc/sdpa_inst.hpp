@@ -116,7 +116,7 @@ int MOTIF_CAT(launch_gda_decode_, MOTIF_SUFFIX)(const SdpaArgs& a, int gc, int w
   if constexpr (std::is_same<MOTIF_ELEM, half_t>::value ||
                 std::is_same<MOTIF_ELEM, bf16_t>::value) {
     const int rc = launch_gda_decode_mfma_16<MOTIF_ELEM>(a, gc, waves, nblocks, s);
-    if (rc != MOTIF_OK) return rc;
+    if (rc != MOTIF_OK || a.nsplit == 1) return rc;  // (one split: no merge launch)
     return launch_gda_decode_merge_d<MOTIF_ELEM, 128>(a, s);
   }
   set_error("gda_decode: no fused variant for this element type");
@@ -140,7 +140,7 @@ int MOTIF_CAT(launch_gda_decode_q_, MOTIF_SUFFIX)(const SdpaArgs& a, int bits, i
                                                  hipStream_t s) {
   if constexpr (!std::is_same<MOTIF_ELEM, float>::value) {  // fp16 and bf16
     const int rc = launch_gda_decode_mfma_q<MOTIF_ELEM>(a, bits, a.group_size, gc, nblocks, s);
-    if (rc != MOTIF_OK) return rc;
+    if (rc != MOTIF_OK || a.nsplit == 1) return rc;  // (one split: no merge launch)
     return launch_gda_decode_merge_d<MOTIF_ELEM, 128>(a, s);
   }
   set_error("gda_decode_q: no fused variant for this element type");

@@ -249,6 +249,15 @@ inline bool tile_softmax_scale_ok(float qscale) {
 // 12.58 / 10.25, 2048 12.74 / 11.03, 3204 13.92 / 13.47, 4096 14.32 / 13.96.
 constexpr int kShortDecodeRows = 4096;
 
+// The fused decode step over at most this many rows runs one split per KV
+// head, whose workgroup applies the epilogue itself: no partials, and one
+// launch instead of two.  A longer chain per workgroup against the merge
+// launch (32 + 8 heads over 8 KV heads, us per step, splits of 64 rows / one
+// split): fp16 cache, batch 1, 130 rows 10.7 / 8.3, 256 rows 10.6 / 9.6, 384
+// rows 10.7 / 11.7; batch 16, 256 rows 17.2 / 12.6; q4 256 rows 12.3 / 10.7;
+// bf16 over q8 256 rows 14.4 / 13.9, 384 rows 14.5 / 15.6.
+constexpr int kOneSplitRows = 256;
+
 // Plan of the packed-cache matrix-core kernel (head_dim 128, fp16): 4-wave
 // workgroups at one wave per SIMD, one per CU.
 constexpr int kSdpaMfmaQD = 128;
