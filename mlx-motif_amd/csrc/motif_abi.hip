@@ -170,14 +170,21 @@ PrefillPlan plan_prefill(int B, int Hq, int Hkv, int S_q, int kv_len, int D) {
   const int bh = B * Hkv;
   // 8 waves (128 virtual heads per block, two waves per SIMD) from 512
   // virtual heads per KV head on, even if the row splits that fill the GPU
-  // then need the merge launch; 4 below (measured, 32 q-heads over 8 KV
-  // heads: 512 rows over 3716 157 -> 127 us, 256 rows 93 -> 76 us; at 64
-  // rows 4 waves were faster, 41 vs 47 us, now even).  Slabs of fewer than
+  // then need the merge launch (measured, 32 q-heads over 8 KV heads: 512
+  // rows over 3716 157 -> 127 us, 256 rows 93 -> 76 us).  Slabs of fewer than
   // 64 heads (17..63 over 2048+ rows) take 8 waves too: the waves past the
   // heads only copy tiles, and the extra copy issuers help a read-bound
   // block (5 rows over 32768: 38.0 vs 40.3 us; over 16000: 23.3 vs 24.9; 8
   // rows over 16000: 23.8 vs 25.5).
-  p.waves = GV >= 512 || GV < kPrefillMinHeads ? 8 : 4;
+  // One block's worth of heads (up to 128) takes 8 waves as well, since two
+  // 4-wave blocks read the rows twice (4 / 8 waves, 8 KV heads, fp16: 128
+  // heads over 600 rows 15.7 / 14.8 us, over 3500 25.3 / 20.7); between, 8
+  // waves from 28000 (head, row) pairs per CU on, where the halved block
+  // count is worth more than the shorter splits (400 heads over 1500 rows
+  // 23.6 / 23.1 us, over 2200 28.4 / 26.0, over 8000 67.3 / 47.2; 256 over
+  // 1500 19.2 / 23.2, over 3500 27.4 / 26.6, over 8000 42.7 / 34.8).
+  const bool long_rows = (long)B * Hkv * GV * kv_len >= 28000L * cus;
+  p.waves = GV >= 512 || GV <= 128 || long_rows ? 8 : 4;
   if (tuning().waves_per_wg) p.waves = tuning().waves_per_wg;
   // Two column blocks per wave (256 virtual heads per 8-wave block: each
   // K/V fragment read from LDS feeds twice the MFMAs) from 2048 virtual heads

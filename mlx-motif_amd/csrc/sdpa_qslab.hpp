@@ -341,7 +341,8 @@ __device__ inline half2_t scale_pair(uint32_t bits, int e, half2_t h2) {
     const _Float16 v = (_Float16)ldexpf(__builtin_bit_cast(float, bits << 16), -e);
     return half2_t{v, v};
   } else {
-    return as_h2((bits & 0xFFFFu) | (bits << 16)) * h2;
+    const _Float16 v = __builtin_bit_cast(_Float16, (uint16_t)bits);
+    return half2_t{v, v} * h2;
   }
 }
 
