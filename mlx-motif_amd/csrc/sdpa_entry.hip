@@ -363,12 +363,13 @@ static GdaDecodeLayout gda_decode_layout(int B, int Hkv, int G1, int G2, int kv_
   const bool short4 = kv_len <= kShortDecodeRows;
   L.plan = plan_sdpa(B, Hkv, Hkv, 1, kv_len, D, 1, short4 ? 4 : 0, short4 ? 1 : 0);
   L.plan_q = plan_sdpa(B, Hkv, Hkv, 1, kv_len, D, 1, kSdpaMfmaQWaves, kSdpaMfmaQWgsPerCu);
-  // Short contexts in one split: no partials and no merge launch.
-  if (kv_len <= kOneSplitRows && tuning().rows_per_split == 0 && tuning().min_wgs == 0) {
-    for (SdpaPlan* p : {&L.plan, &L.plan_q}) {
-      p->nsplit = 1;
-      p->rows_per_split = (kv_len + 127) / 128 * 128;
-    }
+  // One tile per wave of an 8-wave workgroup: one split, no merge launch (64
+  // rows or fewer are one split of 4 waves already).
+  if (kv_len > 64 && kv_len <= kOneSplitRows && G1 + G2 <= 8 && tuning().rows_per_split == 0 &&
+      tuning().min_wgs == 0 && tuning().waves_per_wg == 0) {
+    L.plan.nsplit = 1;
+    L.plan.rows_per_split = kOneSplitRows;
+    L.plan.waves = 8;
   }
   const int ns = L.plan.nsplit > L.plan_q.nsplit ? L.plan.nsplit : L.plan_q.nsplit;
   const size_t prow = (size_t)B * Hkv * (G1 + G2);

@@ -249,14 +249,19 @@ inline bool tile_softmax_scale_ok(float qscale) {
 // 12.58 / 10.25, 2048 12.74 / 11.03, 3204 13.92 / 13.47, 4096 14.32 / 13.96.
 constexpr int kShortDecodeRows = 4096;
 
-// The fused decode step over at most this many rows runs one split per KV
-// head, whose workgroup applies the epilogue itself: no partials, and one
-// launch instead of two.  A longer chain per workgroup against the merge
-// launch (32 + 8 heads over 8 KV heads, us per step, splits of 64 rows / one
-// split): fp16 cache, batch 1, 130 rows 10.7 / 8.3, 256 rows 10.6 / 9.6, 384
-// rows 10.7 / 11.7; batch 16, 256 rows 17.2 / 12.6; q4 256 rows 12.3 / 10.7;
-// bf16 over q8 256 rows 14.4 / 13.9, 384 rows 14.5 / 15.6.
-constexpr int kOneSplitRows = 256;
+// The fused decode step over at most 16 rows per wave of one workgroup runs
+// one split per KV head, whose workgroup applies the epilogue itself: no
+// partials, and one launch instead of two.  On the 16-bit cache with up to 8
+// columns that is an 8-wave workgroup and 128 rows (32 + 8 heads over 8 KV
+// heads, fp16, 64-row splits and the merge launch / one split: batch 1, 65
+// rows 10.6 / 9.0 us, 128 rows 10.7 / 9.6; batch 16, 128 rows 12.6 / 11.1);
+// elsewhere 64 rows, which a 4-wave workgroup holds (64 rows of q4 8.65 us,
+// 32-row splits 12.25).  Not past that, though
+// one split is faster up to 256 rows (fp16, 131 rows 10.7 / 8.3 us): a wave's
+// largest softmax weight is exactly 1, so with several tiles per wave fewer of
+// the large weights are exact in fp16, and the error against 64 bits grows
+// (fp16 by 2-5%, q4 and q8 by 15-23%).
+constexpr int kOneSplitRows = 128;
 
 // Plan of the packed-cache matrix-core kernel (head_dim 128, fp16): 4-wave
 // workgroups at one wave per SIMD, one per CU.
