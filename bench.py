@@ -685,7 +685,7 @@ def secondary(torch, lib, dev, steps: int = 50, warm: int = 5) -> dict:
     token's write, at 3204 over 48 layer caches, the 5-row verify
     slabs over 32768 rows (fp16 and q8), the 512-row prefill chunk over 3716
     rows and a 12.7B layer's 512-row chunk at offset 3204 from the
-    projections (RoPE + 4-slot write + both passes in one launch)."""
+    projections (RoPE + 4-slot write, then both passes)."""
     from mlx_motif.kernels import gda_prefill_attention_from_proj
 
     from mlx_motif.kernels import gda_post_split, polynorm
@@ -865,8 +865,8 @@ def run_extra(torch, lib, dev, args):
         del calls, keep
         torch.cuda.empty_cache()
     # a 12.7B layer's prefill chunk from the projections: 512 rows at offset
-    # 3204 (and a first chunk at offset 0), RoPE + cache write + origin
-    # (32 heads) and noise (8 heads) passes in one launch, against
+    # 3204 (and a first chunk at offset 0), RoPE + cache write, then the
+    # origin (32 heads) and noise (8 heads) passes in one launch, against
     # rope_split4 + two multi-row calls
     from mlx_motif.kernels import gda_prefill_attention_from_proj, rope_split4, sdpa_dual_v_rows
     g3 = torch.Generator(device=dev)

@@ -14,7 +14,7 @@ import) routes every wrapper to its reference.
     rope.py      — rope_split4 (RoPE + q/k/v head split + 4-slot cache write
                    in one launch; the reference uses rope() and reshapes)
     prefill.py   — gda_prefill_attention_from_proj (a layer's prefill chunk:
-                   RoPE, cache write and both dual-V passes in one launch)
+                   RoPE and cache write, then both dual-V passes)
 """
 
 from .attention import (

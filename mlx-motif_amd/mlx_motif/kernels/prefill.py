@@ -8,9 +8,9 @@ into q1/q2 (``model.py:669-679``) and, on the k_ratio-1 fallback, runs four
 ``mx.fast.scaled_dot_product_attention`` calls with the causal mask whose
 concatenated outputs are the origin and noise attention
 (``model.py:769-797``), which then feed ``gda_post_split``.  Here that is one
-attention launch (``motif_gda_prefill_proj``; a split merge follows when the
-rows are split): q roped in registers, the chunk's K/V tiles taken from the
-projections and roped in LDS, the chunk's rows written into the 4-slot cache.
+call (``motif_gda_prefill_proj``): a launch for RoPE, the head split and the
+chunk's rows of the 4-slot cache, one for the attention of both passes, and a
+split merge when rows are split.
 """
 
 from __future__ import annotations
@@ -55,7 +55,7 @@ def gda_prefill_attention_from_proj(q_proj, k_proj, v_proj, caches, offset: int,
     offset + S - 1`` are written (k roped at positions ``offset + s``).
     Returns ``(attn_origin, attn_noise)``: (B, q_groups*gr, S, 2D) and (B,
     q_groups, S, 2D), each ``[softmax(q k^T * scale) V1 || ... V2]`` with
-    query row s seeing cache rows ``[0, offset + s]``.  One launch
+    query row s seeing cache rows ``[0, offset + s]``.  One native call
     (``motif_gda_prefill_proj``) where the kernel takes the shape (fp16/bf16,
     D = 128), else ``rope_split4`` and two ``sdpa_dual_v_rows`` calls.
     ``rope_scaling``: None, or a default / linear config
